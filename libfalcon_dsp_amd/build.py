@@ -20,7 +20,7 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 ROOT = os.path.dirname(HERE)
 CSRC = os.path.join(HERE, "csrc")
 HIP_SOURCES = [os.path.join(CSRC, f)
-               for f in ("fdsp_kernels.hip", "fdsp_chan_groups.hip", "fdsp_chan_seg.hip", "fdsp_capi.hip", "fdsp_serve.hip", "fdsp_fm.hip",
+               for f in ("fdsp_kernels.hip", "fdsp_fir.hip", "fdsp_chan_groups.hip", "fdsp_chan_seg.hip", "fdsp_capi.hip", "fdsp_serve.hip", "fdsp_fm.hip",
                          "fdsp_iir.hip", "fdsp_predefined.hip")]
 PREDEFINED_INC = os.path.join(CSRC, "fdsp_predefined_table.inc")
 HIP_LIB = os.path.join(HERE, "libfdsp_hip.so")

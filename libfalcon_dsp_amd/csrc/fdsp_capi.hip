@@ -713,6 +713,7 @@ extern "C" int fdsp_resampler_apply(fdsp_resampler_t h, const fdsp_cf32 *in, siz
 // ===========================================================================
 struct fdsp_fir_s {
     uint32_t m = 0;
+    bool real = true;  // every tap's imaginary part is zero
     DevBuf d_taps, d_hist[2], d_in, d_out;
     uint32_t parity = 0;
     hipStream_t stream = nullptr;
@@ -726,6 +727,8 @@ extern "C" int fdsp_fir_create(const fdsp_cf32 *coeffs, uint32_t n_coeffs, fdsp_
     if (!h)
         return set_err(FDSP_ENOMEM, "host allocation failed");
     h->m = n_coeffs;
+    for (uint32_t k = 0; k < n_coeffs; ++k)
+        h->real &= coeffs[k].im == 0.f;
     const size_t hbytes = (size_t)(n_coeffs > 1 ? n_coeffs - 1 : 1) * sizeof(float2);
     int rc = h->d_taps.ensure(n_coeffs * sizeof(float2));
     if (!rc)
@@ -787,8 +790,9 @@ int fir_device(fdsp_fir_t h, const T *d_in, size_t n, T *d_out, fdsp_stream_t st
         return set_err(FDSP_EINVAL, "null buffers");
     if (int rc = check_chunk(n, 1))
         return rc;
-    hipError_t e = launch_fir(d_in, (uint32_t)n, h->d_taps.as<float2>(), h->m, h->d_hist[h->parity].as<float2>(),
-                              h->d_hist[h->parity ^ 1].as<float2>(), d_out, pick(h->stream, stream));
+    hipError_t e = launch_fir(d_in, (uint32_t)n, h->d_taps.as<float2>(), h->m, h->real,
+                              h->d_hist[h->parity].as<float2>(), h->d_hist[h->parity ^ 1].as<float2>(), d_out,
+                              pick(h->stream, stream));
     if (e == hipErrorInvalidValue)
         return set_err(FDSP_ERANGE, "fir: %u taps exceed the LDS tile", h->m);
     HIP_TRY(e);

@@ -139,9 +139,10 @@ hipError_t launch_resampler(const float2 *in, uint32_t n, uint64_t p, uint32_t u
                             float2 *out, uint32_t count, hipStream_t s);
 
 // FIR with complex taps over one chunk; hist_in/hist_out hold m-1 samples
-// (float whatever the sample type); TI, TO as for launch_nco_multi
+// (float whatever the sample type); TI, TO as for launch_nco_multi; real:
+// every tap's imaginary part is zero
 template <typename TI, typename TO>
-hipError_t launch_fir(const TI *in, uint32_t n, const float2 *taps, uint32_t m, const float2 *hist_in,
+hipError_t launch_fir(const TI *in, uint32_t n, const float2 *taps, uint32_t m, bool real, const float2 *hist_in,
                       float2 *hist_out, TO *out, hipStream_t s);
 
 // FIR bank with real taps, n_chan channels of n samples each

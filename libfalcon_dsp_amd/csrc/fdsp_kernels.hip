@@ -395,92 +395,6 @@ hipError_t launch_resampler(const float2 *in, uint32_t n, uint64_t p, uint32_t u
 }
 
 // ---------------------------------------------------------------------------
-// FIR with complex taps, one stream
-// (reference falcon_dsp_fir_filter::apply, .cc:177-243; CUDA __fir_filter,
-//  _cuda.cu:102-187). y[n] = sum_k h[k] x[n-k], accumulated k = 0..M-1.
-// Input window and taps staged in LDS.
-// ---------------------------------------------------------------------------
-template <int kBlock, bool kTapsLds, typename TI, typename TO>
-__global__ __launch_bounds__(kBlock) void fir_kernel(const TI *__restrict__ in, uint32_t n,
-                                                     const float2 *__restrict__ taps, uint32_t m,
-                                                     const float2 *__restrict__ hist_in,
-                                                     float2 *__restrict__ hist_out, TO *__restrict__ out,
-                                                     uint32_t tile)
-{
-    extern __shared__ __align__(16) unsigned char smem[];
-    const uint32_t hlen = m - 1;
-    if (blockIdx.x == 0) {
-        for (uint32_t t = threadIdx.x; t < hlen; t += kBlock) {
-            const int64_t i = (int64_t)n - hlen + t;
-            hist_out[t] = i >= 0 ? sample_f32(in[i]) : hist_in[hlen + i];
-        }
-    }
-    const uint32_t o0 = blockIdx.x * tile;
-    const uint32_t nt = min(tile, n - o0);
-    float2 *xs = reinterpret_cast<float2 *>(smem);
-    float2 *ts = xs + tile + hlen;
-    const int64_t lo = (int64_t)o0 - hlen;
-    for (uint32_t t = threadIdx.x; t < nt + hlen; t += kBlock) {
-        const int64_t i = lo + t;
-        xs[t] = i >= 0 ? sample_f32(in[i]) : hist_in[hlen + i];
-    }
-    if (kTapsLds)
-        for (uint32_t t = threadIdx.x; t < m; t += kBlock)
-            ts[t] = taps[t];
-    __syncthreads();
-    const float2 *g = kTapsLds ? ts : taps;
-    for (uint32_t q = threadIdx.x; q < nt; q += kBlock) {
-        const float2 *xw = xs + q + hlen;  // xw[-k] = x[o0 + q - k]
-        float2 acc = make_float2(0.f, 0.f);
-        if constexpr (std::is_same<TO, short2>::value) {
-            // integer output: the reference's rounding, product then sum, no
-            // fused multiply-add (falcon_dsp_fir_filter.cc:208-230)
-            for (uint32_t k = 0; k < m; ++k) {
-                const float2 p = cmul_ref(xw[-(int32_t)k], g[k]);
-                {
-#pragma clang fp contract(off)
-                    acc.x = acc.x + p.x;
-                    acc.y = acc.y + p.y;
-                }
-            }
-        } else {
-            for (uint32_t k = 0; k < m; ++k) {
-                const float2 x = xw[-(int32_t)k];
-                const float2 h = g[k];
-                // complex<float> product added to the accumulator, reference order
-                acc.x += x.x * h.x - x.y * h.y;
-                acc.y += x.x * h.y + x.y * h.x;
-            }
-        }
-        sample_put(out + o0 + q, acc);
-    }
-}
-
-template <typename TI, typename TO>
-hipError_t launch_fir(const TI *in, uint32_t n, const float2 *taps, uint32_t m, const float2 *hist_in,
-                      float2 *hist_out, TO *out, hipStream_t s)
-{
-    constexpr int kBlock = 256;
-    const uint32_t tile = 2048;
-    const bool taps_lds = m <= 2048;
-    const size_t lds = (size_t)(tile + m - 1) * sizeof(float2) + (taps_lds ? m * sizeof(float2) : 0);
-    if (lds > 64 * 1024)
-        return hipErrorInvalidValue;
-    const uint32_t blocks = (n + tile - 1) / tile;
-    if (taps_lds)
-        hipLaunchKernelGGL((fir_kernel<kBlock, true, TI, TO>), dim3(blocks), dim3(kBlock), lds, s, in, n, taps, m,
-                           hist_in, hist_out, out, tile);
-    else
-        hipLaunchKernelGGL((fir_kernel<kBlock, false, TI, TO>), dim3(blocks), dim3(kBlock), lds, s, in, n, taps, m,
-                           hist_in, hist_out, out, tile);
-    return hipGetLastError();
-}
-template hipError_t launch_fir<float2, float2>(const float2 *, uint32_t, const float2 *, uint32_t, const float2 *,
-                                               float2 *, float2 *, hipStream_t);
-template hipError_t launch_fir<short2, short2>(const short2 *, uint32_t, const float2 *, uint32_t, const float2 *,
-                                               float2 *, short2 *, hipStream_t);
-
-// ---------------------------------------------------------------------------
 // FIR bank, real taps, many channels (compute-bound FP32 VALU kernel).
 // blockIdx.y is the channel. Each thread keeps kR consecutive outputs in
 // registers and slides a kR+kR-1 sample register window down the input, so
