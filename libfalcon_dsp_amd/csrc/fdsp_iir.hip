@@ -1202,32 +1202,46 @@ extern "C" int fdsp_iir1_apply(fdsp_iir1_t h, const float *in, size_t n, float *
 
 // ===========================================================================
 // IIR bank: many independent streams through one filter. One stream's exact
-// recurrence is sequential, so each stream runs on one lane. A block of four
-// waves owns 64 streams and walks their samples in tiles of kBankT as a
-// pipeline: in phase q, wave 0 runs the recurrence of tile q-2 (lane =
-// stream, in place over the tile's b-parts), while waves 1-3 write tile q's
-// inputs (loaded in phase q-1) and its carried inputs into LDS, issue the
-// loads of tile q+1, form the b-parts of tile q-1 and store the outputs of
-// tile q-3, all with accesses coalesced along each stream's row. A barrier
-// ends each phase. The arithmetic is that of the single-stream kernels (mac,
+// recurrence is sequential, so the streams run side by side on the lanes. A
+// block owns 32 streams and walks their samples in tiles of 32 as a pipeline
+// of four waves; in phase q
+//   role 0    runs the recurrence of tile q-2, in place over its b-parts,
+//   roles 1,2 form the b-parts of tile q-1, half of its samples each,
+//   role 3    puts tile q's inputs into LDS (loaded from memory in phase q-3),
+//             loads tile q+3 and stores tile q-3's outputs.
+// A barrier ends each phase. LDS holds real and imaginary parts in rows of
+// their own, row 2 s + part for stream s, and a lane runs one part of one
+// stream (row = lane). With real coefficients the parts are independent; with
+// complex ones the lane takes the other part's outputs from its neighbour. The
+// arithmetic is that of the single-stream kernels (mac,
 // fb_step): outputs equal the reference's loop (falcon_dsp_iir_filter.cc:
 // 235-396) run on each stream, up to the sign of zero.
+//
+// Bound by role 0's chain with up to about 4096 streams (a 4th-order filter
+// with real coefficients is eight operations a sample, five of them one after
+// another: about 44 cycles with a tile's LDS reads and barrier), beyond by the
+// memory traffic. 8192 samples a stream, 4th order: 172 us at 64 streams, 174
+// at 1024, 184 at 4096, about 530 at 16384 (4.1 TB/s), against 849 to 884 us
+// when a block owned 64 streams, one lane ran both parts of each and three
+// waves shared the rest of the work in tiles of 16 samples. Order 16, complex
+// coefficients, 4097 samples: 488 us against 1066 (one lane a stream: 1094).
+// What it took: loads in straight runs (233 us at 1024 streams with a choice
+// of two forms), the b-taps unrolled with the window in registers (213 us with
+// a window read for each four taps), three tiles' loads in flight (4096
+// streams: 262 us with two; four spill registers). Reading role 0's next half
+// tile ahead of the barrier, and moving row pointers on instead of forming
+// them, measured no faster.
 // ===========================================================================
 namespace {
 
-constexpr uint32_t kBankT = 16;          // samples per tile
-constexpr uint32_t kBankMaxB = 17;       // b taps: up to 16 carried inputs (LDS below 64 KiB)
+constexpr uint32_t kBankS = 32;             // streams a block
+constexpr uint32_t kBankT = 32;             // samples a tile
+constexpr uint32_t kBankB = 16;             // samples a batch of rows' 16-byte LDS accesses
+constexpr uint32_t kBankRow = kBankT + 4;   // LDS row: the lanes' 16-byte accesses fall in distinct banks
+constexpr uint32_t kBankAhead = 3;          // tiles whose loads are in flight
+constexpr uint32_t kBankMaxB = 17;          // b taps: up to 16 carried inputs
 constexpr uint32_t kBankH = kBankMaxB - 1;  // carried-input slots per stream in the state array
-constexpr uint32_t kBankVRow = kBankT + 1;  // LDS row of b-parts / outputs (odd)
-constexpr uint32_t kBankProd = 192;      // producer threads (waves 1-3)
-constexpr uint32_t kBankPer = (64 * kBankT + kBankProd - 1) / kBankProd;  // tile entries per producer
-
-// LDS row of inputs: h carried inputs, then the tile (odd length)
-__host__ __device__ constexpr uint32_t bank_xrow(uint32_t h) { return (h + kBankT) | 1u; }
-__host__ __device__ constexpr size_t bank_lds_bytes(uint32_t h)
-{
-    return (size_t)(2 * 64 * bank_xrow(h) + 3 * 64 * kBankVRow) * sizeof(float2);
-}
+static_assert(kBankH + 8 <= kBankT, "a tile's b-parts reach back into one earlier tile");
 
 struct BankLaunch {
     const void *in;
@@ -1239,159 +1253,350 @@ struct BankLaunch {
     float2 *yh;       // per stream kMaxFb carried outputs, newest first
 };
 
-template <uint32_t T> __device__ __forceinline__ float2 bank_load(const void *p, size_t i)
+typedef float bank_row[kBankRow];
+
+// one or two consecutive samples of a row: as they lie in memory, their parts
+// in the LDS rows, and from one to the other
+template <uint32_t T> using BankOne = typename std::conditional<T == kSampleCf32, float2, uint32_t>::type;
+template <uint32_t T> using BankPair = typename std::conditional<T == kSampleCf32, float4, uint2>::type;
+
+__device__ __forceinline__ float2 one_values(uint32_t v)
 {
-    if constexpr (T == kSampleCf32) {
-        return static_cast<const float2 *>(p)[i];
-    } else {
-        const short2 s = static_cast<const short2 *>(p)[i];
-        return make_float2((float)s.x, (float)s.y);
-    }
+    return make_float2((float)(short)(v & 0xffffu), (float)(short)(v >> 16));
 }
-template <uint32_t T> __device__ __forceinline__ void bank_store(void *p, size_t i, float2 v)
+__device__ __forceinline__ void one_bits(float2 v, uint32_t &o)
 {
-    if constexpr (T == kSampleCf32)
-        static_cast<float2 *>(p)[i] = v;
-    else
-        static_cast<short2 *>(p)[i] = make_short2(i16_trunc(v.x), i16_trunc(v.y));
+    o = (uint32_t)(uint16_t)i16_trunc(v.x) | ((uint32_t)(uint16_t)i16_trunc(v.y) << 16);
+}
+__device__ __forceinline__ void to_rows(float2 v, float *re, float *im)
+{
+    *re = v.x;
+    *im = v.y;
+}
+__device__ __forceinline__ void to_rows(uint32_t v, float *re, float *im) { to_rows(one_values(v), re, im); }
+__device__ __forceinline__ void to_rows(float4 v, float *re, float *im)
+{
+    *reinterpret_cast<float2 *>(re) = make_float2(v.x, v.z);
+    *reinterpret_cast<float2 *>(im) = make_float2(v.y, v.w);
+}
+__device__ __forceinline__ void to_rows(uint2 v, float *re, float *im)
+{
+    const float2 a = one_values(v.x), b = one_values(v.y);
+    to_rows(make_float4(a.x, a.y, b.x, b.y), re, im);
+}
+__device__ __forceinline__ void from_rows(const float *re, const float *im, float2 &v) { v = make_float2(*re, *im); }
+__device__ __forceinline__ void from_rows(const float *re, const float *im, uint32_t &v)
+{
+    one_bits(make_float2(*re, *im), v);
+}
+__device__ __forceinline__ void from_rows(const float *re, const float *im, float4 &v)
+{
+    const float2 r = *reinterpret_cast<const float2 *>(re), i = *reinterpret_cast<const float2 *>(im);
+    v = make_float4(r.x, i.x, r.y, i.y);
+}
+__device__ __forceinline__ void from_rows(const float *re, const float *im, uint2 &v)
+{
+    const float2 r = *reinterpret_cast<const float2 *>(re), i = *reinterpret_cast<const float2 *>(im);
+    one_bits(make_float2(r.x, i.x), v.x);
+    one_bits(make_float2(r.y, i.y), v.y);
 }
 
-template <int P, bool RA, uint32_t TS>
-__global__ __launch_bounds__(256) void iir_bank_kernel(BankLaunch g, Fb<P> fb)
+template <uint32_t N> __device__ __forceinline__ void row_read(const float *p, float (&v)[N])
 {
-    extern __shared__ float2 bank_lds[];
-    const uint32_t h = g.nb - 1, xrow = bank_xrow(h);
-    float2 *xt = bank_lds;                     // [2][64][xrow]: tile q in xt + (q % 2) * 64 * xrow
-    float2 *vt = bank_lds + 2 * 64 * xrow;     // [3][64][kBankVRow]: tile q in vt + (q % 3) * 64 * kBankVRow
-    const uint32_t tid = threadIdx.x, s0 = blockIdx.x * 64;
-    const uint32_t rows = min(64u, g.n_streams - s0);
+#pragma unroll
+    for (uint32_t i = 0; i < N; i += 4) {
+        const float4 w = *reinterpret_cast<const float4 *>(p + i);
+        v[i] = w.x;
+        v[i + 1] = w.y;
+        v[i + 2] = w.z;
+        v[i + 3] = w.w;
+    }
+}
+template <uint32_t N> __device__ __forceinline__ void row_write(float *p, const float (&v)[N])
+{
+#pragma unroll
+    for (uint32_t i = 0; i < N; i += 4)
+        *reinterpret_cast<float4 *>(p + i) = make_float4(v[i], v[i + 1], v[i + 2], v[i + 3]);
+}
+
+// four samples of a row from position `at` (a multiple of 4) of the tile at
+// cur; below 0 they end the row's previous tile
+__device__ __forceinline__ void row_four(const float *cur, const float *prev, int32_t at, float *w)
+{
+    const float4 v = *reinterpret_cast<const float4 *>(at >= 0 ? cur + at : prev + (int32_t)kBankT + at);
+    w[0] = v.x;
+    w[1] = v.y;
+    w[2] = v.z;
+    w[3] = v.w;
+}
+
+// one part of a complex product, rounded as cmul_ref rounds it: `own` and
+// `other` are the factor's parts, hx the coefficient's real part, hy its
+// imaginary part with the sign it has in this part
+__device__ __forceinline__ float part_product(float own, float other, float hx, float hy)
+{
+#pragma clang fp contract(off)
+    return own * hx + other * hy;
+}
+
+// one part of a stream's recurrence: fb_step on it, the other part's outputs
+// from the neighbouring lane
+template <int P, bool RA> struct BankState {
+    float own[P];
+    float other[RA ? 1 : P], aside[RA ? 1 : P];
+    __device__ __forceinline__ float step(float v, const Fb<P> &fb)
+    {
+#pragma clang fp contract(off)
+        if constexpr (RA) {
+            return fb_step<P, false>(v, own, fb);
+        } else {
+            float y = v;
+#pragma unroll
+            for (int k = 0; k < P; ++k)
+                y = y - part_product(own[k], other[k], fb.a[k].x, aside[k]);
+#pragma unroll
+            for (int k = P - 1; k > 0; --k) {
+                own[k] = own[k - 1];
+                other[k] = other[k - 1];
+            }
+            own[0] = y;
+            other[0] = __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(y), 0xB1, 0xF, 0xF, false));
+            return y;
+        }
+    }
+};
+
+// PAIR: the rows' sample pairs are aligned to their size, in and out
+template <int P, bool RA, uint32_t TS, bool PAIR>
+__global__ __launch_bounds__(256, 2) void iir_bank_kernel(BankLaunch g, Fb<P> fb)
+{
+    // [tile % 3][2 * stream + part][sample]: inputs; b-parts, then outputs
+    __shared__ __align__(16) bank_row xt[3][2 * kBankS], vt[3][2 * kBankS];
+    const uint32_t tid = threadIdx.x, lane = tid & 63, part = lane & 1, s0 = blockIdx.x * kBankS;
+    // blocks 256 apart share a CU: rotated, their recurrences take different SIMDs
+    const uint32_t role = (__builtin_amdgcn_readfirstlane(tid >> 6) + blockIdx.x / 256) & 3;
+    const uint32_t rows = min(kBankS, g.n_streams - s0);
     const uint32_t nt = (g.n + kBankT - 1) / kBankT;
     const auto tile_cnt = [&](uint32_t q) { return min(kBankT, g.n - q * kBankT); };
-    __shared__ float2 bsh[kBankMaxB];  // the b taps, read by all lanes at once
-    if (tid < g.nb)
-        bsh[tid] = g.b[tid];
-    float2 st[P];  // wave 0: the stream's carried outputs, newest first
-    // waves 1-3: the inputs of the next two tiles in flight (tile q in
-    // pf[q % 2]), so each load has two phases to land
-    float2 pf0[kBankPer], pf1[kBankPer];
-    if (tid < 64) {
-#pragma unroll
-        for (int k = 0; k < P; ++k)
-            st[k] = tid < rows ? g.yh[(size_t)(s0 + tid) * kMaxFb + k] : make_float2(0.f, 0.f);
+    // the carried inputs end the tile before the first
+    for (uint32_t e = tid; e < kBankS * kBankH; e += 256) {
+        const uint32_t r = e / kBankH, k = e % kBankH;
+        const float2 v = r < rows ? g.xh[(size_t)(s0 + r) * kBankH + k] : make_float2(0.f, 0.f);
+        xt[2][2 * r][kBankT - kBankH + k] = v.x;
+        xt[2][2 * r + 1][kBankT - kBankH + k] = v.y;
     }
-    const uint32_t p = tid - 64;  // producer index (waves 1-3)
-    const auto load_tile = [&](uint32_t q, float2 (&pf)[kBankPer]) {
-        const uint32_t t0 = q * kBankT, cnt = tile_cnt(q);
+    __syncthreads();
+
+    if (role == 0) {
+        const uint32_t sr = lane / 2;
+        BankState<P, RA> st;
 #pragma unroll
-        for (uint32_t i = 0; i < kBankPer; ++i) {
-            const uint32_t e = i * kBankProd + p, r = e / kBankT, c = e % kBankT;
-            pf[i] = r < rows && c < cnt ? bank_load<TS>(g.in, (size_t)(s0 + r) * g.in_stride + t0 + c)
-                                        : make_float2(0.f, 0.f);
+        for (int k = 0; k < P; ++k) {
+            const float2 y = sr < rows ? g.yh[(size_t)(s0 + sr) * kMaxFb + k] : make_float2(0.f, 0.f);
+            st.own[k] = part ? y.y : y.x;
+            if constexpr (!RA) {
+                st.other[k] = part ? y.x : y.y;
+                st.aside[k] = part ? fb.a[k].y : -fb.a[k].y;
+            }
         }
-    };
-    if (tid >= 64 && nt > 0)
-        load_tile(0, pf0);
-    if (tid >= 64 && nt > 1)
-        load_tile(1, pf1);
-    const auto phase = [&](uint32_t q, float2 (&pf)[kBankPer]) {
-        if (tid < 64) {
-            // the recurrence of tile q - 2 along the lane's stream
-            if (q >= 2 && q - 2 < nt && tid < rows) {
+        for (uint32_t q = 0; q < nt + 3; ++q) {
+            if (q >= 2 && q - 2 < nt) {
                 const uint32_t cnt = tile_cnt(q - 2);
-                float2 *vr = vt + ((q - 2) % 3) * 64 * kBankVRow + tid * kBankVRow;
-#pragma unroll 4
-                for (uint32_t t = 0; t < cnt; ++t)
-                    vr[t] = fb_step<P, true, RA>(vr[t], st, fb);
-            }
-        } else {
-            if (q < nt) {
-                // tile q's inputs after its carried inputs: the last h of
-                // (carried inputs, tile q - 1), or the state array for tile 0
-                float2 *xq = xt + (q % 2) * 64 * xrow;
-                const uint32_t cnt = tile_cnt(q);
+                float *v = vt[(q - 2) % 3][lane];
+                if (cnt == kBankT) {
+                    float x[kBankB], y[kBankB];
+                    row_read(v, x);
+                    row_read(v + kBankB, y);
 #pragma unroll
-                for (uint32_t i = 0; i < kBankPer; ++i) {
-                    const uint32_t e = i * kBankProd + p, r = e / kBankT, c = e % kBankT;
-                    if (r < 64 && c < cnt)
-                        xq[r * xrow + h + c] = pf[i];
-                }
-                for (uint32_t e = p; e < 64 * h; e += kBankProd) {
-                    const uint32_t r = e / h, k = e - r * h;
-                    if (r < rows)
-                        xq[r * xrow + k] = q == 0 ? g.xh[(size_t)(s0 + r) * kBankH + kBankH - h + k]
-                                                  : xt[((q - 1) % 2) * 64 * xrow + r * xrow + tile_cnt(q - 1) + k];
-                }
-                if (q + 2 < nt)
-                    load_tile(q + 2, pf);
-            }
-            if (q >= 1 && q - 1 < nt) {
-                // b-parts of tile q - 1: ((0 + b0 x[n]) + b1 x[n-1]) + ...,
-                // the lane's entries side by side, one tap at a time
-                const float2 *xq = xt + ((q - 1) % 2) * 64 * xrow;
-                float2 *vq = vt + ((q - 1) % 3) * 64 * kBankVRow;
-                const uint32_t cnt = tile_cnt(q - 1);
-                float2 acc[kBankPer];
-                uint32_t base[kBankPer];
+                    for (uint32_t t = 0; t < kBankB; ++t)
+                        x[t] = st.step(x[t], fb);
+                    row_write(v, x);
 #pragma unroll
-                for (uint32_t i = 0; i < kBankPer; ++i) {
-                    const uint32_t e = i * kBankProd + p, r = min(e / kBankT, 63u), c = e % kBankT;
-                    acc[i] = make_float2(0.f, 0.f);
-                    base[i] = r * xrow + h + c;
-                }
-                for (uint32_t k = 0; k < g.nb; ++k) {
-                    const float2 bk = bsh[k];
-#pragma unroll
-                    for (uint32_t i = 0; i < kBankPer; ++i)
-                        acc[i] = mac<true, RA>(acc[i], xq[base[i] - k], bk);
-                }
-#pragma unroll
-                for (uint32_t i = 0; i < kBankPer; ++i) {
-                    const uint32_t e = i * kBankProd + p, r = e / kBankT, c = e % kBankT;
-                    if (r < rows && c < cnt)
-                        vq[r * kBankVRow + c] = acc[i];
+                    for (uint32_t t = 0; t < kBankB; ++t)
+                        y[t] = st.step(y[t], fb);
+                    row_write(v + kBankB, y);
+                } else {
+                    for (uint32_t t = 0; t < cnt; ++t)
+                        v[t] = st.step(v[t], fb);
                 }
             }
-            if (q >= 3 && q - 3 < nt) {
-                // outputs of tile q - 3
-                const float2 *vq = vt + ((q - 3) % 3) * 64 * kBankVRow;
-                const uint32_t t0 = (q - 3) * kBankT, cnt = tile_cnt(q - 3);
-#pragma unroll
-                for (uint32_t i = 0; i < kBankPer; ++i) {
-                    const uint32_t e = i * kBankProd + p, r = e / kBankT, c = e % kBankT;
-                    if (r < rows && c < cnt)
-                        bank_store<TS>(g.out, (size_t)(s0 + r) * g.out_stride + t0 + c, vq[r * kBankVRow + c]);
-                }
-            }
+            __syncthreads();
         }
-        __syncthreads();
-    };
-    for (uint32_t q = 0; q < nt + 3; q += 2) {
-        phase(q, pf0);
-        if (q + 1 < nt + 3)
-            phase(q + 1, pf1);
-    }
-    // carried state: the last h inputs of (carried inputs, last tile), and the outputs
-    if (tid < 64 && tid < rows) {
-        const float2 *xl = xt + ((nt - 1) % 2) * 64 * xrow + tid * xrow + tile_cnt(nt - 1);
-        for (uint32_t k = 0; k < h; ++k)
-            g.xh[(size_t)(s0 + tid) * kBankH + kBankH - h + k] = xl[k];
+        if (sr < rows) {
 #pragma unroll
-        for (int k = 0; k < P; ++k)
-            g.yh[(size_t)(s0 + tid) * kMaxFb + k] = st[k];
+            for (int k = 0; k < P; ++k)
+                reinterpret_cast<float *>(g.yh + (size_t)(s0 + sr) * kMaxFb + k)[part] = st.own[k];
+        }
+    } else if (role < 3) {
+        const int32_t t0 = (int32_t)((role - 1) * kBankB);
+        // the taps, in scalar registers
+        const auto bp = (const __attribute__((address_space(4))) float *)reinterpret_cast<const float *>(g.b);
+        float2 b[kBankMaxB];
+#pragma unroll
+        for (uint32_t k = 0; k < kBankMaxB; ++k)
+            b[k] = k < g.nb ? make_float2(bp[2 * k], bp[2 * k + 1]) : make_float2(0.f, 0.f);
+        for (uint32_t q = 0; q < nt + 3; ++q) {
+            if (q >= 1 && q - 1 < nt) {
+                // ((0 + b0 x[n]) + b1 x[n-1]) + ..., four taps a step
+                const uint32_t c = (q - 1) % 3, p = (q + 1) % 3;  // this tile's slot, the previous one's
+                // the batch's window, sample t0 - 20 + i at w[i]: four taps
+                // reach four samples further back, read before the taps ahead
+                // of them are summed
+                constexpr uint32_t kBack = (kBankMaxB + 3) / 4 * 4;
+                float w[kBack + kBankB], z[RA ? 4 : kBack + kBankB];  // z: the other part's
+                const auto read = [&](int32_t i) {
+                    row_four(xt[c][lane], xt[p][lane], t0 - (int32_t)kBack + i, w + i);
+                    if constexpr (!RA)
+                        row_four(xt[c][lane ^ 1], xt[p][lane ^ 1], t0 - (int32_t)kBack + i, z + i);
+                };
+                float acc[kBankB];
+#pragma unroll
+                for (uint32_t i = 0; i < kBankB; ++i)
+                    acc[i] = 0.f;
+                const auto tap = [&](uint32_t k) {
+#pragma unroll
+                    for (uint32_t i = 0; i < kBankB; ++i) {
+                        const uint32_t at = kBack + i - k;
+                        if constexpr (RA)
+                            acc[i] = mac<false>(acc[i], w[at], b[k]);
+                        else
+                            acc[i] = acc[i] + part_product(w[at], z[at], b[k].x, part ? b[k].y : -b[k].y);
+                    }
+                };
+#pragma unroll
+                for (uint32_t i = 0; i < kBankB + 4; i += 4)
+                    read((int32_t)(kBack - 4 + i));
+#pragma unroll
+                for (uint32_t k0 = 0; k0 < kBankMaxB; k0 += 4) {
+                    if (k0 >= g.nb)
+                        break;
+                    if (k0 + 4 < kBankMaxB)
+                        read((int32_t)kBack - 8 - (int32_t)k0);
+                    if (k0 + 4 <= g.nb) {
+#pragma unroll
+                        for (uint32_t kk = 0; kk < 4; ++kk)
+                            if (k0 + kk < kBankMaxB)
+                                tap(k0 + kk);
+                    } else {
+#pragma unroll
+                        for (uint32_t kk = 0; kk < 3; ++kk)
+                            if (k0 + kk < kBankMaxB && k0 + kk < g.nb)
+                                tap(k0 + kk);
+                    }
+                }
+                row_write(vt[c][lane] + t0, acc);
+            }
+            __syncthreads();
+        }
+    } else {
+        // Round i of the lane: stream i kRows + r0, sample(s) c0 of the tile.
+        // Whole tiles are loaded ahead, unconditionally (past the last
+        // whole tile, that one again) and in one straight run: a load under a
+        // condition, or from one of two places, was waited for where it was
+        // issued. What the rows past the last stream load is not used.
+        using One = BankOne<TS>;
+        using Item = typename std::conditional<PAIR, BankPair<TS>, One>::type;
+        constexpr uint32_t kItem = PAIR ? 2 : 1, kRows = 64 * kItem / kBankT, kIo = kBankS / kRows;
+        const uint32_t r0 = lane / (kBankT / kItem), c0 = kItem * (lane % (kBankT / kItem));
+        const One *in = static_cast<const One *>(g.in) + (size_t)s0 * g.in_stride;
+        One *out = static_cast<One *>(g.out) + (size_t)s0 * g.out_stride;
+        const uint32_t whole = g.n / kBankT;
+        const auto load_tile = [&](uint32_t q, Item (&pf)[kIo]) {
+            const One *p = in + min(q, whole - 1) * kBankT + c0;
+#pragma unroll
+            for (uint32_t i = 0; i < kIo; ++i)
+                pf[i] = *reinterpret_cast<const Item *>(p + (size_t)min(i * kRows + r0, rows - 1) * g.in_stride);
+        };
+        const auto store_tile = [&](uint32_t q) {
+            const uint32_t cnt = tile_cnt(q), t = q % 3;
+            One *o = out + q * kBankT;
+            if (cnt == kBankT && rows == kBankS) {
+#pragma unroll
+                for (uint32_t i = 0; i < kIo; ++i) {
+                    const uint32_t r = i * kRows + r0;
+                    Item y;
+                    from_rows(&vt[t][2 * r][c0], &vt[t][2 * r + 1][c0], y);
+                    *reinterpret_cast<Item *>(o + (size_t)r * g.out_stride + c0) = y;
+                }
+            } else {
+                for (uint32_t e = lane; e < rows * kBankT; e += 64) {
+                    const uint32_t r = e / kBankT, c = e % kBankT;
+                    One y;
+                    from_rows(&vt[t][2 * r][c], &vt[t][2 * r + 1][c], y);
+                    if (c < cnt)
+                        o[(size_t)r * g.out_stride + c] = y;
+                }
+            }
+        };
+        const auto phase = [&](uint32_t q, Item (&pf)[kIo]) {
+#pragma unroll
+            for (uint32_t i = 0; i < kIo; ++i) {
+                const uint32_t r = i * kRows + r0;
+                to_rows(pf[i], &xt[q % 3][2 * r][c0], &xt[q % 3][2 * r + 1][c0]);
+            }
+            load_tile(q + kBankAhead, pf);
+            if (q >= 3)
+                store_tile(q - 3);
+            __syncthreads();
+        };
+        uint32_t q = 0;
+        if (whole > 0) {
+            Item pf[kBankAhead][kIo];
+#pragma unroll
+            for (uint32_t u = 0; u < kBankAhead; ++u)
+                load_tile(u, pf[u]);
+            for (; q + kBankAhead <= whole; q += kBankAhead) {
+#pragma unroll
+                for (uint32_t u = 0; u < kBankAhead; ++u)
+                    phase(q + u, pf[u]);
+            }
+#pragma unroll
+            for (uint32_t u = 0; u + 1 < kBankAhead; ++u)
+                if (q < whole)
+                    phase(q++, pf[u]);
+        }
+        for (; q < nt + 3; ++q) {
+            if (q < nt) {  // the last tile, when partial
+                for (uint32_t e = lane; e < rows * kBankT; e += 64) {
+                    const uint32_t r = e / kBankT, c = e % kBankT;
+                    if (c < tile_cnt(q))
+                        to_rows(in[(size_t)r * g.in_stride + q * kBankT + c], &xt[q % 3][2 * r][c],
+                                &xt[q % 3][2 * r + 1][c]);
+                }
+            }
+            if (q >= 3)
+                store_tile(q - 3);
+            __syncthreads();
+        }
+        // the last kBankH of (carried inputs, chunk): tiles nt-1 and nt-2
+        const int32_t end = (int32_t)tile_cnt(nt - 1);
+        for (uint32_t e = lane; e < kBankS * kBankH; e += 64) {
+            const uint32_t r = e / kBankH, k = e % kBankH;
+            const int32_t at = end - (int32_t)kBankH + (int32_t)k;
+            const uint32_t t = at >= 0 ? (nt - 1) % 3 : (nt + 1) % 3, c = at >= 0 ? at : (int32_t)kBankT + at;
+            if (r < rows)
+                g.xh[(size_t)(s0 + r) * kBankH + k] = make_float2(xt[t][2 * r][c], xt[t][2 * r + 1][c]);
+        }
     }
 }
 
 template <int P, uint32_t TS> hipError_t launch_bank_p(const BankLaunch &g, const float2 *a, bool ra, hipStream_t s)
 {
+    const uintptr_t bytes = sizeof(BankPair<TS>);
+    const bool pair = reinterpret_cast<uintptr_t>(g.in) % bytes == 0 && g.in_stride % 2 == 0 &&
+                      reinterpret_cast<uintptr_t>(g.out) % bytes == 0 && g.out_stride % 2 == 0;
     Fb<P> fb;
     for (int k = 0; k < P; ++k)
         fb.a[k] = a[k];
-    const dim3 grid((g.n_streams + 63) / 64);
-    const size_t lds = bank_lds_bytes(g.nb - 1);
-    if (ra)
-        hipLaunchKernelGGL((iir_bank_kernel<P, true, TS>), grid, dim3(256), lds, s, g, fb);
+    const dim3 grid((g.n_streams + kBankS - 1) / kBankS);
+    if (ra && pair)
+        hipLaunchKernelGGL((iir_bank_kernel<P, true, TS, true>), grid, dim3(256), 0, s, g, fb);
+    else if (ra)
+        hipLaunchKernelGGL((iir_bank_kernel<P, true, TS, false>), grid, dim3(256), 0, s, g, fb);
+    else if (pair)
+        hipLaunchKernelGGL((iir_bank_kernel<P, false, TS, true>), grid, dim3(256), 0, s, g, fb);
     else
-        hipLaunchKernelGGL((iir_bank_kernel<P, false, TS>), grid, dim3(256), lds, s, g, fb);
+        hipLaunchKernelGGL((iir_bank_kernel<P, false, TS, false>), grid, dim3(256), 0, s, g, fb);
     return hipGetLastError();
 }
 

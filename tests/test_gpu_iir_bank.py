@@ -110,3 +110,34 @@ def test_bank_rejects_bad_arguments():
         fd.IirBank([1.0], [1.0], 0)
     with pytest.raises(fd.FdspError):
         fd.IirBank([1.0], [0.0, 1.0], 4)  # a[0] == 0
+
+
+@pytest.mark.parametrize("sample", ["cf32", "ci16"])
+@pytest.mark.parametrize("nb,nfb,cplx,streams,offset,si,so", [(1, 1, False, 31, 0, 98, 98), (5, 4, False, 33, 1, 97, 99),
+                                                            (17, 16, False, 32, 0, 99, 98), (16, 3, True, 1, 1, 98, 97),
+                                                            (17, 15, True, 34, 0, 97, 97)])
+def test_bank_tile_edges_and_alignment(nb, nfb, cplx, streams, offset, si, so, sample):
+    # chunks around the 32-sample tile, one after another, on rows whose sample
+    # pairs are aligned to their size or not, blocks of 32 streams full and partial
+    u = np.random.default_rng(nb + nfb + streams)
+    b, a = random_filter(u, nb, nfb, cplx, 1.0)
+    bank, refs = fd.IirBank(b, a, streams), _oracles(b, a, streams)
+    dt, st = (fd.CI16 if sample == "ci16" else np.dtype(np.complex64)), fd.Stream()
+    d_in, d_out = fd.DeviceBuffer(streams * si + 1, dt), fd.DeviceBuffer(streams * so + 1, dt)
+    for n in (1, 15, 16, 31, 32, 33, 63, 64, 65, 97):
+        x = (u.standard_normal((streams, si, 2)) * 2000).round().astype(np.int16)
+        z = (x[..., 0] + 1j * x[..., 1]).astype(np.complex64) / 777
+        flat = np.zeros(streams * si + 1, dt)
+        flat[offset:offset + streams * si] = x.reshape(-1, 2).view(fd.CI16)[:, 0] if sample == "ci16" else z.reshape(-1)
+        d_in.upload(flat)
+        fn = fd.lib().fdsp_iir_bank_apply_ci16_device if sample == "ci16" else fd.lib().fdsp_iir_bank_apply_device
+        assert fn(bank.h, d_in.at(offset), n, si, d_out.at(offset), so, st.h) == 0
+        st.sync()
+        got = d_out.download()[offset:offset + streams * so].reshape(streams, so)[:, :n]
+        for s in range(streams):
+            if sample == "ci16":
+                want = refs[s].apply_ci16(x[s, :n])
+                have = np.stack([got[s]["re"], got[s]["im"]], -1)
+            else:
+                want, have = refs[s].apply(z[s, :n]), got[s]
+            np.testing.assert_array_equal(have, want, err_msg=f"n {n} stream {s}")
