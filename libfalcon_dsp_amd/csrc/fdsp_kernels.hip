@@ -498,19 +498,29 @@ __global__ __launch_bounds__(kBlock) void fir_bank_kernel(const float2 *__restri
 // imaginary parts of the samples are two GEMMs sharing A. A block stages
 // its input window and the zero-padded taps in LDS; each wave accumulates
 // kFbG column groups of 16 blocks.
+//
+// Bound by the matrix cores on long filters, by the memory traffic on short
+// ones. 256 channels x 2^17 samples, back to back, with one, two, three and
+// four groups a wave: 512 taps 574 (eight waves a block), 547, 536 and 569 us
+// (128 of the 153 TFLOP/s that a large FP32 matrix product reaches); 101 taps
+// 185, 173, 161 and 252 us; 32 taps 126, 129, 119 and 205 us (4.5 TB/s): more
+// groups read fewer A operands, fewer leave LDS for more blocks a CU, whose
+// loads and stores then run under other blocks' products.
 typedef float fb_floatx4 __attribute__((ext_vector_type(4)));
-constexpr uint32_t kFbG = 4, kFbWaves = 4;
-constexpr uint32_t kFbTile = kFbWaves * kFbG * 256;  // outputs per block
+constexpr uint32_t kFbWaves = 4;
+constexpr uint32_t fb_tile(uint32_t groups) { return kFbWaves * groups * 256; }  // outputs per block
 // one padding sample per 16, so the 16 columns of a B read (16 samples apart)
 // fall in distinct banks
 __host__ __device__ __forceinline__ uint32_t fb_pad(uint32_t q) { return q + (q >> 4); }
 
+template <uint32_t kFbG>
 __global__ __launch_bounds__(kFbWaves * 64) void fir_bank_mfma_kernel(
     const float2 *__restrict__ in, uint32_t n, uint64_t in_stride, const float *__restrict__ taps, uint32_t m,
     uint32_t kp, const float2 *__restrict__ hist_in, float2 *__restrict__ hist_out, float2 *__restrict__ out,
     uint64_t out_stride)
 {
     extern __shared__ __align__(16) unsigned char smem[];
+    constexpr uint32_t kFbTile = fb_tile(kFbG);
     float2 *xs = reinterpret_cast<float2 *>(smem);
     const uint32_t span = kFbTile + kp - 16;
     float *hs = reinterpret_cast<float *>(xs + fb_pad(span) + 1);  // kp + 16 taps
@@ -626,13 +636,33 @@ hipError_t launch_fir_bank(const float2 *in, uint32_t n, uint64_t in_stride, con
                            uint64_t out_stride, hipStream_t s)
 {
     {
-        // the matrix-core form whenever its window and taps fit the LDS
+        // The matrix-core form whenever its window and taps fit the LDS: three
+        // column groups a wave where that gives at least 16 blocks a CU, else
+        // two (256 channels x 8192 samples, 768 and 1024 blocks: 512 taps 43.2
+        // and 40.1 us, 32 taps 11.5 and 10.0), one where two leave less than
+        // two blocks a CU.
         const uint32_t kp = (m + 15 + 3) / 4 * 4;
-        const size_t lds = (size_t)(fb_pad(kFbTile + kp - 16) + 1) * sizeof(float2) + (kp + 16) * sizeof(float);
-        if (lds <= 64 * 1024) {
-            dim3 grid((n + kFbTile - 1) / kFbTile, n_chan);
-            hipLaunchKernelGGL(fir_bank_mfma_kernel, grid, dim3(kFbWaves * 64), lds, s, in, n, in_stride, taps, m,
-                               kp, hist_in, hist_out, out, out_stride);
+        const auto lds_of = [&](uint32_t groups) {
+            return (size_t)(fb_pad(fb_tile(groups) + kp - 16) + 1) * sizeof(float2) + (kp + 16) * sizeof(float);
+        };
+        const auto blocks_of = [&](uint32_t groups) {
+            return (uint64_t)((n + fb_tile(groups) - 1) / fb_tile(groups)) * n_chan;
+        };
+        uint32_t groups = blocks_of(3) >= 4096 ? 3u : blocks_of(2) >= 512 ? 2u : 1u;
+        while (groups > 1 && lds_of(groups) > 64 * 1024)
+            --groups;
+        if (lds_of(groups) <= 64 * 1024) {
+            const dim3 grid((n + fb_tile(groups) - 1) / fb_tile(groups), n_chan);
+#define FDSP_FB_LAUNCH(G)                                                                                       \
+    hipLaunchKernelGGL(fir_bank_mfma_kernel<G>, grid, dim3(kFbWaves * 64), lds_of(G), s, in, n, in_stride, taps, m, \
+                       kp, hist_in, hist_out, out, out_stride)
+            if (groups == 3)
+                FDSP_FB_LAUNCH(3);
+            else if (groups == 2)
+                FDSP_FB_LAUNCH(2);
+            else
+                FDSP_FB_LAUNCH(1);
+#undef FDSP_FB_LAUNCH
             return hipGetLastError();
         }
     }

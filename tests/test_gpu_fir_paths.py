@@ -40,6 +40,25 @@ def test_float_chunks(m, lens, real):
         at += n
 
 
+@pytest.mark.parametrize("n_chan,m,n", [(3, 1, 1), (5, 4, 1023), (3, 17, 1025), (300, 33, 4097), (600, 64, 2049),
+                                        (1400, 20, 9001), (4, 4300, 5000), (4, 5100, 4000)])
+def test_bank_groups_a_wave(n_chan, m, n):
+    # one, two and three column groups a wave (blocks of 1024, 2048 and 3072
+    # outputs), ragged last blocks, the longest windows of the matrix form and
+    # the VALU form beyond them, the history carried into a second chunk
+    rng = np.random.default_rng(m)
+    taps = (rng.standard_normal((n_chan, m)) / np.sqrt(m)).astype(np.float32)
+    x = cwgn(11 + m, n_chan * 2 * n).reshape(n_chan, 2 * n)
+    bank = fd.FirBank(taps)
+    got = np.concatenate([bank.apply(x[:, :n]), bank.apply(x[:, n:])], axis=1)
+    tol = 10 * np.sqrt(m + 4) * U
+    for c in {0, 1, n_chan // 2, n_chan - 1}:
+        size = 1 << int(2 * n + m).bit_length()
+        want = np.fft.ifft(np.fft.fft(x[c].astype(np.complex128), size) * np.fft.fft(taps[c].astype(float), size))
+        scale = np.sqrt(np.mean(np.abs(x[c]) ** 2) * np.sum(taps[c].astype(float) ** 2))
+        assert np.max(np.abs(got[c] - want[:2 * n])) <= tol * scale, (n_chan, m, n, c)
+
+
 @pytest.mark.parametrize("n", [3000, 140_000])
 @pytest.mark.parametrize("real", [False, True])
 def test_non_finite_samples_reach_their_windows_only(n, real):
