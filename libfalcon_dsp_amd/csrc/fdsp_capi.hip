@@ -1318,10 +1318,19 @@ float bf16_to_float(uint16_t b)
     return f;
 }
 
-// Work plan of the segment-major FP32 kernel. Channels with up 1, at most 32
-// taps and the same down form MFMA groups of 2..8 (a larger set of one down
-// splits into near-equal groups); every other channel is a one-channel VALU
-// group. Each channel's modulated taps are padded in front to its window
+// Whether n channels of one down are faster as an MFMA group (wide: with
+// discriminator tails or 64-tap windows) than as VALU channels. A wide
+// sub-tile of 15 or 16 rows costs about what a VALU channel's batch of 63 or
+// 64 does, whatever the number of its channels (up to eight). 4 x 10^6 inputs
+// at down 80, calls back to back: 2 tails of 64 taps 17.6 us on VALU and 20.1
+// in a group, 3 of 32 taps 13.7 and 14.8, 7 of 32 taps 20.1 and 15.8, 12 of 64
+// taps 39.5 and 27.0.
+bool mfma_pays(size_t n, bool wide) { return n >= (wide ? 4u : 2u); }
+
+// Work plan of the segment-major FP32 kernel. Channels with up 1 and the same
+// down, window (32 or 64) and tail form MFMA groups of 2..8 (a larger set
+// splits into near-equal groups) where mfma_pays says so; every other channel
+// is a one-channel VALU group. Each channel's modulated taps are padded in front to its window
 // (32 or 64) per filter phase. Leaves use_seg false when a window exceeds 64
 // taps or the plan exceeds the kernel's limits (the group kernel then runs).
 void build_seg_plan(fdsp_channelizer_s *h, const std::vector<float2> &taps)
@@ -1368,20 +1377,21 @@ void build_seg_plan(fdsp_channelizer_s *h, const std::vector<float2> &taps)
                 ptaps.push_back(taps[s.taps_off + ph * k.cpp + t]);
         }
     }
-    // MFMA groups by down
+    // MFMA groups by down, window and tail
     std::vector<bool> done(C, false);
     std::vector<SegGroup> mfma, valu;
     for (uint32_t c = 0; c < C; ++c) {
         const ChanHost &k = h->ch[c];
-        if (done[c] || k.up != 1 || k.cpp > 32 || k.tail)
+        if (done[c] || k.up != 1)
             continue;
+        const uint32_t win = h->stat[c].win;
         std::vector<uint32_t> same;
         for (uint32_t d = c; d < C; ++d) {
             const ChanHost &o = h->ch[d];
-            if (!done[d] && o.up == 1 && o.cpp <= 32 && !o.tail && o.down == k.down)
+            if (!done[d] && o.up == 1 && h->stat[d].win == win && !o.tail == !k.tail && o.down == k.down)
                 same.push_back(d);
         }
-        if (same.size() < 2)
+        if (!mfma_pays(same.size(), win == 64 || k.tail))
             continue;
         const size_t n_g = (same.size() + kMfmaMaxChan - 1) / kMfmaMaxChan;
         for (size_t g = 0, at = 0; g < n_g; ++g) {
@@ -1391,7 +1401,8 @@ void build_seg_plan(fdsp_channelizer_s *h, const std::vector<float2> &taps)
             gr.m = (uint32_t)take;
             gr.up = 1;
             gr.down = k.down;
-            gr.win = 32;
+            gr.win = win;
+            gr.tail = k.tail;
             gr.btab = (uint32_t)h->seg_btab.size();
             for (size_t i = 0; i < take; ++i) {
                 gr.chan[i] = same[at + i];
@@ -1401,7 +1412,7 @@ void build_seg_plan(fdsp_channelizer_s *h, const std::vector<float2> &taps)
             // t = g + 4(s/2), part s%2 (0 real, 1 imaginary); column 2c gives
             // channel c's real output (Gr xr - Gi xi), 2c+1 its imaginary
             // output (Gi xr + Gr xi)
-            for (uint32_t st = 0; st < 16; ++st)
+            for (uint32_t st = 0; st < win / 2; ++st)
                 for (uint32_t lane = 0; lane < 64; ++lane) {
                     const uint32_t col = lane % 16, t = lane / 16 + 4 * (st / 2), part = st % 2;
                     float v = 0.f;
@@ -1482,9 +1493,9 @@ SegArgs seg_args(const fdsp_channelizer_s *h, const fdsp_cf32 *d_in, uint32_t n,
     a.out16 = true;
     for (const ChanStatic &st : h->stat)
         a.out16 = a.out16 && reinterpret_cast<uintptr_t>(st.out) % 16 == 0;
-    a.tails = false;
+    a.wide = false;
     for (const SegGroup &g : h->seg_groups)
-        a.tails = a.tails || g.tail != 0;
+        a.wide = a.wide || g.tail != 0 || (g.kind == kSegMfma && g.win == 64);
     return a;
 }
 

@@ -26,7 +26,9 @@
 //         sample g+4j at K step 2j and its imaginary part at step 2j+1. The
 //         modulated taps are the B operand in the same K order: channel c's
 //         real output in column 2c, its imaginary output in 2c+1. A sub-tile
-//         is 16 outputs of every channel of the group.
+//         is 16 outputs of every channel of the group. Windows of 33 to 64
+//         taps take 32 K steps. Channels with a discriminator tail form groups
+//         of their own, whose sub-tiles overlap by one output.
 //   VALU  one channel (any up), window of at most 64 taps: one output per
 //         lane, taps zero-padded in front to kW = 32 or 64. With up 1 the taps
 //         are wavefront-uniform scalar loads; with up > 1 each lane reads the
@@ -369,6 +371,133 @@ __device__ __forceinline__ void mfma_group(const SegDev &a, cptr<SegGroup> gr, c
 }
 
 // ---------------------------------------------------------------------------
+// MFMA group with discriminator tails or a 64-tap window: this wave's
+// sub-tiles st, st + kWaves, ... < n_st
+// ---------------------------------------------------------------------------
+// Sub-tile s computes rows 16 s .. 16 s + 15 or, with tails, 15 s - 1 ..
+// 15 s + 14: its row 0 only gives the others their predecessor (the segment's
+// row -1 as for VALU channels, see there). The phasors are evaluated per row in
+// FP64: these groups have few rows a segment.
+//
+// Bound by the sub-tile's MFMA chain and the latencies around it (span load,
+// phasors, angles). 16 tails of 64 taps at down 80 have 26 outputs a segment of
+// 2048 inputs each; as VALU channels (one output a lane, 26 of 64 lanes at
+// work, 16 channels in turn) 2 x 10^6 inputs took 29.8 us, in two groups
+// 14.8 us.
+template <uint32_t kWin>
+__device__ __forceinline__ void mfma_wide_group(const SegDev &a, cptr<SegGroup> gr, bool tail, const ChanRun &run,
+                                                const ChanRun *runs, const SegPos &pos, const float2 *xs,
+                                                uint32_t span_lo, uint32_t st, uint32_t n_st, uint32_t lane)
+{
+    const uint32_t down = gr->down, m = gr->m;
+    const int32_t n_rows = (int32_t)(run.j_hi - run.j_lo);
+    // opaque per call: keeps the group's loads inside the segment
+    asm volatile("" : "+v"(lane));
+    constexpr uint32_t kHalves = kWin / 32;
+    float bv[kHalves][16];
+    {
+        const float *bt = a.btab + gr->btab + lane;
+#pragma unroll
+        for (uint32_t h = 0; h < kHalves; ++h)
+#pragma unroll
+            for (uint32_t s = 0; s < 16; ++s)
+                bv[h][s] = bt[(16 * h + s) * 64];
+    }
+    // lanes and rows as in mfma_group
+    const uint32_t col = lane & 15, g = lane >> 4;
+    const bool odd = col & 1, live = (col >> 1) < m;
+    const uint32_t ci = gr->chan[min(col >> 1, m - 1)];
+    const ChanStatic *csp = a.chans + ci;
+    const uint32_t R = csp->r;
+    const double nu = csp->nu;
+    const uint32_t k_lo = runs[ci].k_lo;
+    const int32_t ro = (int32_t)(4 * g + (odd ? 2u : 0u));
+    const int32_t step = tail ? 15 : 16, row0 = tail ? -1 : 0;
+    // chunk output of a row to compute, clamped to rows whose window is staged
+    const auto output_of = [&](int32_t rr) {
+        const int32_t rc = min(rr, n_rows - 1);
+        return (uint32_t)((int32_t)run.j_lo + (rc < 0 && run.j_lo == 0 ? 0 : rc));
+    };
+    const auto window_of = [&](uint32_t j) { return j * down + run.rho - (kWin - 1) - span_lo; };
+    // the row's output, phased: rollover correction as in finish_out
+    const auto phased = [&](int32_t rr, float2 y) {
+        int32_t k = (int32_t)(k_lo + (uint32_t)rr * down);
+        if (k < 0)
+            k += (int32_t)R;
+        if ((uint32_t)k >= R)
+            k -= (int32_t)R;
+        if (rr < n_rows && (uint32_t)k + 1 < kWin && (rr >= 0 || run.j_lo > 0)) {
+            const float2 *gt = a.ptaps + csp->poff;
+            const float2 wrap_m1 = make_float2(csp->wrap.x - 1.f, csp->wrap.y);
+            const uint32_t q = window_of(output_of(rr));
+            float2 part = make_float2(0.f, 0.f);
+            for (uint32_t t = 0; t + 1 + (uint32_t)k < kWin; ++t)
+                cmac(part, gt[t], xs[slot(q + t, a.km)]);
+            cmac(y, wrap_m1, part);
+        }
+        return cmul(nco_phasor((int64_t)k, nu), y);
+    };
+    for (; st < n_st; st += kWaves) {
+        const int32_t top = row0 + step * (int32_t)st;  // the sub-tile's row 0
+        const float2 *p = xs + slot(window_of(output_of(top + (int32_t)col)) + g, a.km);
+        // a chain for each part of each half window: shorter sums round less
+        floatx4 c = floatx4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (uint32_t h = 0; h < kHalves; ++h) {
+            floatx4 re = floatx4{0.f, 0.f, 0.f, 0.f}, im = re;
+#pragma unroll
+            for (uint32_t t = 0; t < 8; ++t) {
+                const float2 x = p[8 * h + t];
+                re = __builtin_amdgcn_mfma_f32_16x16x4f32(x.x, bv[h][2 * t], re, 0, 0, 0);
+                im = __builtin_amdgcn_mfma_f32_16x16x4f32(x.y, bv[h][2 * t + 1], im, 0, 0, 0);
+            }
+            c += re + im;
+        }
+        float oth[4];
+#pragma unroll
+        for (uint32_t e = 0; e < 4; ++e)
+            oth[e] = __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(c[e]), 0xB1, 0xF, 0xF, false));
+        const int32_t rr = top + ro;  // the lane's rows: rr, rr + 1
+        float2 y0 = phased(rr, odd ? make_float2(oth[2], c[2]) : make_float2(c[0], oth[0]));
+        const float2 y1 = phased(rr + 1, odd ? make_float2(oth[3], c[3]) : make_float2(c[1], oth[1]));
+        const uint32_t j = (uint32_t)((int32_t)run.j_lo + rr);
+        if (!tail) {
+            const gvec2_ptr out = (gvec2_ptr)csp->out;
+            if (live && rr < n_rows)
+                __builtin_nontemporal_store(fvec2{y0.x, y0.y}, out + j);
+            if (live && rr + 1 < n_rows)
+                __builtin_nontemporal_store(fvec2{y1.x, y1.y}, out + j + 1);
+            continue;
+        }
+        const bool overlap = ro == 0;  // row 0 of the sub-tile
+        if (overlap && rr < 0 && run.j_lo == 0 && pos.P > 0)
+            y0 = csp->prev[pos.parity][0];  // the previous chunk's last output
+        // row rr's predecessor: the odd lane's lies in its neighbour, the even
+        // lane's in the odd lane of the rows before
+        const int src = (int)((odd ? lane - 1 : lane - 15) & 63u);
+        const float2 yp = make_float2(__shfl(y1.x, src), __shfl(y1.y, src));
+        if (!live)
+            continue;
+        // (as for VALU channels: the chunk's last output is carried, the
+        // stream's first has no predecessor)
+        const uint32_t drop = pos.P == 0 ? 1u : 0u;
+        const auto emit = [&](uint32_t jj, float2 y, float2 before) {
+            if (jj + 1 == run.j_end)
+                csp->prev[pos.parity ^ 1u][0] = y;
+            if (jj < drop)
+                return;
+            const float2 z = cmul(y, make_float2(before.x, -before.y));
+            __builtin_nontemporal_store(atan2f(z.y, z.x),
+                                        (__attribute__((address_space(1))) float *)csp->out + (jj - drop));
+        };
+        if (!overlap && rr < n_rows)
+            emit(j, y0, yp);
+        if (rr + 1 < n_rows)
+            emit(j + 1, y1, y0);
+    }
+}
+
+// ---------------------------------------------------------------------------
 // VALU channel: batch b of one channel's outputs in the segment
 // ---------------------------------------------------------------------------
 // Without a tail, lane l computes segment row 64 b + l. With a discriminator
@@ -482,12 +611,12 @@ __device__ __forceinline__ void valu_group(const SegDev &a, uint32_t ci, bool ta
 // ---------------------------------------------------------------------------
 // the kernel: one segment per workgroup
 // ---------------------------------------------------------------------------
-// kTails: the plan has discriminator tails. Their code (the angle, the
-// neighbour exchange, the carried sample) sets the kernel's register peak, so
-// plans without them run an instance that leaves it out (fewer VGPRs, more
-// workgroups per CU).
-template <bool kTails>
-__global__ __launch_bounds__(kBlock, 5) void chan_seg_kernel(SegDev a)
+// kWide: the plan has discriminator tails or MFMA groups of 64-tap windows.
+// Their code (the angle, the neighbour exchange, the carried sample; 32 B
+// operands) sets the kernel's register peak, so plans without them run an
+// instance that leaves it out (fewer VGPRs, more workgroups per CU).
+template <bool kWide>
+__global__ __launch_bounds__(kBlock, kWide ? 4 : 5) void chan_seg_kernel(SegDev a)
 {
     const uint32_t km = a.km;
     // dynamic LDS: the transposed span (4 km samples), then one ChanRun per channel
@@ -540,7 +669,9 @@ __global__ __launch_bounds__(kBlock, 5) void chan_seg_kernel(SegDev a)
         if (lane < a.n_groups) {
             const ChanRun &r = runs[g_chan];
             const uint32_t rows = r.j_hi - r.j_lo;
-            cnt = g_kind == kSegMfma ? (rows + 15) / 16 : g_tail ? (rows + 62) / 63 : (rows + 63) / 64;
+            cnt = g_kind == kSegMfma ? (kWide && g_tail ? (rows + 14) / 15 : (rows + 15) / 16)
+                  : g_tail           ? (rows + 62) / 63
+                                     : (rows + 63) / 64;
         }
 #pragma unroll
         for (uint32_t d = 1; d < 64; d <<= 1) {
@@ -634,10 +765,21 @@ __global__ __launch_bounds__(kBlock, 5) void chan_seg_kernel(SegDev a)
         const cptr<SegGroup> gr = groups + g;
         const ChanRun run = runs[gr->chan[0]];
         if (gr->kind == kSegMfma) {
+            if constexpr (kWide) {
+                const bool tail = gr->tail != 0;
+                if (gr->win == 64) {
+                    mfma_wide_group<64>(a, gr, tail, run, runs, pos, xs, span_lo, i - i0, i1 - i0, lane);
+                    continue;
+                }
+                if (tail) {
+                    mfma_wide_group<32>(a, gr, true, run, runs, pos, xs, span_lo, i - i0, i1 - i0, lane);
+                    continue;
+                }
+            }
             mfma_group(a, gr, run, runs, xs, span_lo, i - i0, i1 - i0, lane);
         } else {
             const uint32_t ci = gr->chan[0];
-            const bool tail = kTails && gr->tail != 0;
+            const bool tail = kWide && gr->tail != 0;
             if (gr->win == 32)
                 valu_group<32>(a, ci, tail, run, pos, xs, span_lo, i - i0, i1 - i0, lane);
             else
@@ -653,8 +795,10 @@ __global__ __launch_bounds__(kBlock, 5) void chan_seg_kernel(SegDev a)
         for (uint32_t g = tid; g < a.n_groups; g += kBlock) {
             const SegGroup &gr = a.groups[g];
             if (gr.tail && runs[gr.chan[0]].j_end == 0) {
-                const ChanStatic &c = a.chans[gr.chan[0]];
-                c.prev[parity ^ 1u][0] = c.prev[parity][0];
+                for (uint32_t i = 0; i < (kWide ? gr.m : 1u); ++i) {  // (a group's channels share their rows)
+                    const ChanStatic &c = a.chans[gr.chan[i]];
+                    c.prev[parity ^ 1u][0] = c.prev[parity][0];
+                }
             }
         }
         float2 *hw = parity ? a.histw0 : a.histw1;
@@ -733,7 +877,7 @@ hipError_t launch_chan_seg(const SegArgs &s, hipStream_t stream)
     a.small = geo.small;
     const uint32_t blocks = geo.blocks;
     const size_t lds = geo.lds;
-    if (s.tails)
+    if (s.wide)
         hipLaunchKernelGGL(chan_seg_kernel<true>, dim3(blocks), dim3(kBlock), lds, stream, a);
     else
         hipLaunchKernelGGL(chan_seg_kernel<false>, dim3(blocks), dim3(kBlock), lds, stream, a);

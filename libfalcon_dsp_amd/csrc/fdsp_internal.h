@@ -253,7 +253,7 @@ hipError_t launch_chan_groups(const GroupsArgs &a, hipStream_t s);
 // workgroup per segment of `seg` inputs, staged once with `halo` samples of
 // history before it; records in the order the waves take their work.
 enum : uint32_t {
-    kSegMfma = 0,  // 2..8 channels, up 1, equal down, <= 32 taps: FP32 MFMA sub-tiles of 16 outputs
+    kSegMfma = 0,  // 2..8 channels, up 1, equal down, window and tail: FP32 MFMA sub-tiles of 16 outputs
     kSegValu = 1,  // one channel, window <= 64: one output per lane
 };
 constexpr uint32_t kSegMaxChan = 256;    // channels of one plan at most
@@ -266,8 +266,8 @@ struct SegGroup {
     uint32_t m;        // channels
     uint32_t up, down;
     uint32_t win;      // window (padded taps per phase): 32 or 64
-    uint32_t btab;     // MFMA: offset of the group's B operands (16 x 64 floats)
-    uint32_t tail;     // VALU: the channel ends in the polar discriminator
+    uint32_t btab;     // MFMA: offset of the group's B operands (win/2 x 64 floats)
+    uint32_t tail;     // the channels end in the polar discriminator
     uint32_t pad;
     uint32_t chan[8];  // channel indices
 };
@@ -286,7 +286,7 @@ struct SegArgs {
     uint64_t p;
     uint32_t parity;
     bool out16;
-    bool tails;  // some group ends in the polar discriminator
+    bool wide;  // some group ends in the polar discriminator or is an MFMA group of 64-tap windows
 };
 hipError_t launch_chan_seg(const SegArgs &a, hipStream_t s);
 size_t chan_seg_lds_bytes(uint32_t seg, uint32_t halo, uint32_t n_chan);

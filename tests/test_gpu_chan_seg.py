@@ -19,7 +19,7 @@ import numpy as np
 import pytest
 
 import libfalcon_dsp_amd as fd
-from libfalcon_dsp_amd.signals import cwgn
+from libfalcon_dsp_amd.signals import cwgn, kaiser_sinc
 from libfalcon_dsp_amd.workloads import Chan32, channel
 from oracle import oracle as O
 from tests.helpers import assert_close_rms, chunks, max_err, rms
@@ -254,3 +254,49 @@ def test_fused_discriminator_graph_replays():
             else:
                 assert counts[c] == rs[c].size
                 assert_close_rms(got, rs[c], rms(x), tol=F32_TOL, what=f"replay {k} chan {c}")
+
+
+@pytest.mark.parametrize("n_ch,down,per_up,tail", [(4, 64, 64, True), (5, 80, 32, True), (9, 100, 64, True),
+                                                   (4, 5, 64, True), (5, 63, 20, True), (8, 20, 33, False),
+                                                   (4, 100, 64, False), (4, 7, 40, False)])
+def test_wide_mfma_groups_against_oracle(n_ch, down, per_up, tail):
+    # MFMA groups of tail channels (sub-tiles of 15 rows) and of windows of 33
+    # to 64 taps, where the plan starts to form them: rows per segment below,
+    # at and far above a sub-tile, chunks that emit nothing or one output, the
+    # index rolling over (R of 1e5 to 1e6) inside chunks and windows
+    fs = 1_000_000
+    taps = kaiser_sinc(per_up, 0.5 / down, 8.0).astype(np.complex64)
+    chans = [dict(freq_shift_in_hz=37_000 + 41_003 * c, up_rate=1, down_rate=down, taps=taps) for c in range(n_ch)]
+    if tail:
+        chans = [dict(ch, tail="discriminator") for ch in chans]
+    n = 330_000
+    x = (0.05 * cwgn(61, n)).astype(np.complex128)
+    k = np.arange(n)
+    for c, ch in enumerate(chans):
+        x += np.exp(2j * np.pi * ((-ch["freq_shift_in_hz"] / fs * k) % 1.0)) * (1.0 if c == 0 else 0.05)
+    x = x.astype(np.complex64)
+    g = fd.MultiRateChannelizer(fs, chans)
+    info = g.kernel_info()
+    assert info["kernel"] == "chan_seg_kernel" and info["mfma_groups"] == -(-n_ch // 8) == info["groups"]
+    ref = O.Channelizer(fs, [{q: v for q, v in ch.items() if q != "tail"} for ch in chans])
+    discs = [O.Discriminator() if tail else None for _ in chans]
+    xr = rms(x)
+    for lo, hi in chunks(x.size, [150_000, 3, 1, down, 99_999, 2048, 4097]):
+        ys, rs = g.apply(x[lo:hi]), ref.apply(x[lo:hi])
+        for c in range(n_ch):
+            if not tail:
+                assert ys[c].size == rs[c].size
+                # a tone at the filter's centre: both sums' rounded terms add up to
+                # the signal itself, 2 x 64 of them at u / 2 (one sigma 7e-7) each
+                assert_close_rms(ys[c], rs[c], xr, tol=2 * F32_TOL, what=f"chan {c} [{lo},{hi})")
+                continue
+            want = discs[c].apply(rs[c])
+            assert ys[c].size == want.size, f"chan {c} [{lo},{hi}): {ys[c].size} vs {want.size}"
+            if not want.size:
+                continue
+            # an angle turns by at most the two samples' errors over their sizes
+            z = np.abs(rs[c][rs[c].size - want.size:])
+            before = np.abs(np.concatenate([[np.inf], rs[c]])[rs[c].size - want.size:rs[c].size])
+            d = np.abs(np.angle(np.exp(1j * (ys[c].astype(np.float64) - want))))
+            ok = np.minimum(z, before) > 0.02 * xr
+            assert ok.any() and np.max(d[ok]) <= 4 * F32_TOL / 0.02 + 1e-5, f"chan {c} [{lo},{hi})"
