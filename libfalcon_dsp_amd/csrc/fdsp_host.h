@@ -121,8 +121,10 @@ inline NcoChan make_nco(uint32_t fs, int32_t f)
         c.r = r;
     }
     c.inv_r = 1.0 / (double)c.r;
-    for (int i = 0; i < kNcoSamples; ++i)
+    for (int i = 0; i < kNcoSamples; ++i) {
         c.step[i] = phasor64(c.nu * kNcoOffsets[i]);
+        c.single[i] = phasor64(c.nu * (double)(kNcoSingle * i));
+    }
     c.omega = w;
     return c;
 }

@@ -82,12 +82,17 @@ constexpr int kNcoSamples = 16;
 constexpr uint32_t kNcoOffsets[kNcoSamples] = {0, 1, 128, 129, 256, 257, 384, 385,
                                                512, 513, 640, 641, 768, 769, 896, 897};
 
+// ... and where pairs are not aligned: single samples 64 apart, so a wave's
+// 8-byte accesses each cover 512 consecutive bytes
+constexpr uint32_t kNcoSingle = 64;
+
 struct NcoChan {
     double nu;        // f/fs, signed, revolutions per sample
     double inv_r;     // 1/R
     uint32_t r;       // rollover index R (UINT32_MAX for the identity shift)
     uint32_t tab;     // first entry of this shift's phasor table (kNoTable: none)
     float2 step[kNcoSamples];  // e^{j 2 pi nu o_i}, o = kNcoOffsets: a thread's samples relative to its first
+    float2 single[kNcoSamples];  // the same for o_i = kNcoSingle i
     double omega;     // 2 pi f / fs rad/sample, formed as the reference forms it
 };
 

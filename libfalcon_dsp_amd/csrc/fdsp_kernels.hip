@@ -32,8 +32,16 @@ __device__ __forceinline__ uint64_t ceil_div_u64(uint64_t a, uint64_t b) { retur
 constexpr int kNcoL = kNcoSamples;
 // A thread's samples: pairs 128 apart (lane l: its wave's samples 2l, 2l+1,
 // 128+2l, 129+2l, ...), so each 16-byte load or store instruction of a wave
-// covers 1 KB of consecutive samples; a wave covers 64 kNcoL samples
+// covers 1 KB of consecutive samples; a wave covers 64 kNcoL samples. Where a
+// pair is not aligned to its size in the input and in every output (an odd
+// output stride), single samples 64 apart (lane l: l, 64+l, ...): as pairs they
+// took two accesses of every other sample each (10^6 + 3 samples, 16 shifts:
+// 27.7 us a call against 23.0; 262143: 11.4 and 9.2).
 constexpr const uint32_t (&kNcoOff)[kNcoL] = kNcoOffsets;
+template <bool kVec> __device__ __forceinline__ constexpr uint32_t nco_off(int i)
+{
+    return kVec ? kNcoOff[i] : kNcoSingle * i;
+}
 
 // a thread's samples as whole aligned accesses, one per pair
 __device__ __forceinline__ void load_pairs(const float2 *p, float2 (&x)[kNcoL])
@@ -79,18 +87,24 @@ __global__ __launch_bounds__(256) void nco_multi_kernel(const TI *__restrict__ i
     // blockIdx.y picks the shifts c0 .. c1-1 (cpb per block): small chunks
     // spread their shifts over more blocks, re-reading the input from L2
     const uint32_t c0 = blockIdx.y * cpb, c1 = min(n_chan, c0 + cpb);
-    // the wave's 256 samples, and this lane's first pair in them
-    const uint32_t i0 = (blockIdx.x * blockDim.x + (threadIdx.x & ~63u)) * kNcoL + 2 * (threadIdx.x & 63u);
+    // the wave's 1024 samples, and this lane's first in them
+    const uint32_t i0 =
+        (blockIdx.x * blockDim.x + (threadIdx.x & ~63u)) * kNcoL + (kVec ? 2u : 1u) * (threadIdx.x & 63u);
     if (i0 >= n)
         return;
-    const bool full = i0 + kNcoOff[kNcoL - 1] < n;
+    constexpr uint32_t kLast = nco_off<kVec>(kNcoL - 1);
+    const bool full = i0 + kLast < n;
     float2 x[kNcoL];
     if (kVec && full) {
         load_pairs(in + i0, x);
+    } else if (full) {
+#pragma unroll
+        for (int i = 0; i < kNcoL; ++i)
+            x[i] = sample_f32(in[i0 + nco_off<kVec>(i)]);
     } else {
 #pragma unroll
         for (int i = 0; i < kNcoL; ++i)
-            x[i] = (i0 + kNcoOff[i] < n) ? sample_f32(in[i0 + kNcoOff[i]]) : make_float2(0.f, 0.f);
+            x[i] = (i0 + nco_off<kVec>(i) < n) ? sample_f32(in[i0 + nco_off<kVec>(i)]) : make_float2(0.f, 0.f);
     }
     for (uint32_t c = c0; c < c1; ++c) {
         const double nu = chans[c].nu;
@@ -102,7 +116,7 @@ __global__ __launch_bounds__(256) void nco_multi_kernel(const TI *__restrict__ i
             const uint32_t t0 = chans[c].tab;
 #pragma unroll
             for (int i = 0; i < kNcoL; ++i) {
-                const uint64_t k = k0 + kNcoOff[i] >= r ? k0 + kNcoOff[i] - r : k0 + kNcoOff[i];
+                const uint64_t kn = k0 + nco_off<kVec>(i), k = kn >= r ? kn - r : kn;
                 float2 ph;
                 if (tab && t0 != kNoTable) {
                     ph = tab[t0 + k];
@@ -113,27 +127,33 @@ __global__ __launch_bounds__(256) void nco_multi_kernel(const TI *__restrict__ i
                 }
                 y[i] = cmul_ref(x[i], ph);
             }
-        } else if (k0 + kNcoOff[kNcoL - 1] < r) {
+        } else if (k0 + kLast < r) {
             const float2 base = nco_phasor((int64_t)k0, nu);
+            const float2 *step = kVec ? chans[c].step : chans[c].single;
 #pragma unroll
             for (int i = 0; i < kNcoL; ++i)
-                y[i] = cmul(x[i], cmul(base, chans[c].step[i]));
+                y[i] = cmul(x[i], cmul(base, step[i]));
         } else {
             // the rollover falls inside this thread's samples: index restarts at 0
             const float2 base = nco_phasor((int64_t)k0, nu);
             const float2 basew = nco_phasor((int64_t)k0 - (int64_t)r, nu);
+            const float2 *step = kVec ? chans[c].step : chans[c].single;
 #pragma unroll
             for (int i = 0; i < kNcoL; ++i)
-                y[i] = cmul(x[i], cmul((k0 + kNcoOff[i] < r) ? base : basew, chans[c].step[i]));
+                y[i] = cmul(x[i], cmul((k0 + nco_off<kVec>(i) < r) ? base : basew, step[i]));
         }
         TO *o = out + (uint64_t)c * out_stride;
         if (kVec && full) {
             store_pairs(o + i0, y);
+        } else if (full) {
+#pragma unroll
+            for (int i = 0; i < kNcoL; ++i)
+                sample_put(o + i0 + nco_off<kVec>(i), y[i]);
         } else {
 #pragma unroll
             for (int i = 0; i < kNcoL; ++i)
-                if (i0 + kNcoOff[i] < n)
-                    sample_put(o + i0 + kNcoOff[i], y[i]);
+                if (i0 + nco_off<kVec>(i) < n)
+                    sample_put(o + i0 + nco_off<kVec>(i), y[i]);
         }
     }
 }
@@ -154,9 +174,10 @@ hipError_t launch_nco_multi(const TI *in, uint32_t n, uint64_t start, const NcoC
     const uint32_t groups = min(n_chan, max(1u, target / blocks));
     const uint32_t cpb = (n_chan + groups - 1) / groups;
     const dim3 grid(blocks, (n_chan + cpb - 1) / cpb);
-    // 16-byte accesses of sample pairs: every channel's output must start 16-byte aligned
-    const bool vec = ((reinterpret_cast<uintptr_t>(in) | reinterpret_cast<uintptr_t>(out)) % 16 == 0) &&
-                     (out_stride * sizeof(TO)) % 16 == 0;
+    // accesses of sample pairs: the input and every channel's output must start aligned to a pair
+    const bool vec = reinterpret_cast<uintptr_t>(in) % (2 * sizeof(TI)) == 0 &&
+                     reinterpret_cast<uintptr_t>(out) % (2 * sizeof(TO)) == 0 &&
+                     (n_chan == 1 || out_stride % 2 == 0);
     if (vec)
         hipLaunchKernelGGL((nco_multi_kernel<true, TI, TO>), grid, dim3(256), 0, s, in, n, start, chans, n_chan, out,
                            out_stride, tab, cpb);

@@ -123,3 +123,32 @@ def test_set_state_continues_the_stream():
     np.testing.assert_array_equal(yb, ya)
     assert_close_rms(yb, r, rms(x))
     assert b.samples_handled() == int(ref.samples_handled)
+
+
+@pytest.mark.parametrize("n,stride,offset", [(1, 1, 0), (1023, 1023, 0), (1025, 1026, 0), (64_001, 64_001, 1),
+                                             (99_999, 100_000, 1), (250_001, 250_003, 0)])
+def test_single_sample_accesses_equal_pairs(n, stride, offset):
+    # odd output strides and inputs off a pair's alignment take accesses of
+    # single samples: the same outputs as an aligned handle's within the two
+    # roundings of a sample's phasor, int16 ones bit for bit, across rollovers
+    fs, shifts = 1_000_000, [333_333, -7, 1]
+    u = np.random.default_rng(n)
+    xi = (u.standard_normal((n + 1, 2)) * 5000).round().astype(np.int16)
+    x = (xi[:, 0] + 1j * xi[:, 1]).astype(np.complex64)
+    s = fd.Stream()
+    even = n + (n & 1)
+    for data, dt, call in ((x, np.dtype(np.complex64), "apply_device"), (xi.view(fd.CI16)[:, 0], fd.CI16, "apply_ci16_device")):
+        a, b = fd.FreqShift(fs, shifts), fd.FreqShift(fs, shifts)
+        d_in, d_off = fd.DeviceBuffer.from_array(data[:n].copy()), fd.DeviceBuffer(n + 1, dt)
+        d_off.upload(np.concatenate([data[:offset], data[:n], data[n:n + 1 - offset]]))
+        d_a, d_b = fd.DeviceBuffer(3 * even, dt), fd.DeviceBuffer(3 * stride, dt)
+        for _ in range(2):  # the second chunk starts in the middle of a period
+            getattr(a, call)(d_in, n, d_a, even, s)
+            getattr(b, call)(d_off, n, d_b, stride, s, in_offset=offset)
+        s.sync()
+        want = d_a.download().reshape(3, even)[:, :n]
+        got = d_b.download().reshape(3, stride)[:, :n]
+        if dt == fd.CI16:
+            np.testing.assert_array_equal(got, want)
+        else:
+            assert np.max(np.abs(got - want)) <= 8 * 2.0 ** -24 * np.max(np.abs(x))

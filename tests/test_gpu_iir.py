@@ -231,3 +231,33 @@ def test_reset_after_apply_on_a_caller_stream():
     g.apply_device(d_in, 5000, yb, s)
     s.sync()
     np.testing.assert_array_equal(ya.download(5000), yb.download(5000))
+
+
+@pytest.mark.parametrize("real_in", [False, True])
+@pytest.mark.parametrize("order,cutoff,extra", [(1, 0.3, 0), (2, 0.05, 0), (3, 0.2, 13), (4, 0.1, 0), (6, 0.12, 2),
+                                                (8, 0.3, 8), (8, 0.3, 9)])
+def test_scanned_segments_round_as_the_sequential_loop(order, cutoff, extra, real_in):
+    # unverified segments started from a scan (real coefficients, order <= 8,
+    # at most 17 b taps; 18 take the warm-up form): chunks around a segment (16
+    # or 32 samples) and around a block's outputs, the state carried between
+    # them. The result's error against 64 bits is that of the sequential float
+    # loop: its rounding noise through the same filter, so about the same norm.
+    from scipy.signal import butter, lfilter
+    b, a = butter(order, cutoff)
+    b = np.convolve(b, np.hanning(extra + 2)[1:-1]) if extra else b
+    b, a = b.astype(np.float32), a.astype(np.float32)
+    lens = [1, 15, 16, 17, 31, 33, 700, 831, 832, 833, 927, 928, 929, 991, 993, 1, 4000, 30_011]
+    x = cwgn(50 + order, sum(lens))
+    x = x.real.copy() if real_in else x
+    want = lfilter(b.astype(float), a.astype(float), x.astype(float if real_in else complex))
+    g, o = fd.IirFilter(b, a), O.Iir(b, a)
+    g.set_exact(False)
+    got, seq, lo = [], [], 0
+    for n in lens:
+        c = x[lo:lo + n]
+        got.append(g.apply_f32(c) if real_in else g.apply(c))
+        seq.append(o.apply_f32(c) if real_in else o.apply(c))
+        lo += n
+    e_got = np.linalg.norm(np.concatenate(got) - want)
+    e_seq = np.linalg.norm(np.concatenate(seq) - want)
+    assert e_got <= 2 * e_seq + 1e-7 * np.linalg.norm(want), (e_got, e_seq)
