@@ -101,24 +101,31 @@ template <int P> struct Fb {
 };
 
 // input i >= 0 of the chunk
-template <uint32_t TIN, bool C> __device__ __forceinline__ Val<C> load_in(const IirLaunch &g, int32_t i)
+template <uint32_t TIN> __device__ __forceinline__ float2 chunk_sample(const IirLaunch &g, int32_t i)
 {
-    float2 v;
     if constexpr (TIN == kSampleCf32)
-        v = static_cast<const float2 *>(g.x)[i];
+        return static_cast<const float2 *>(g.x)[i];
     else if constexpr (TIN == kSampleF32)
-        v = make_float2(static_cast<const float *>(g.x)[i], 0.f);
+        return make_float2(static_cast<const float *>(g.x)[i], 0.f);
     else if constexpr (TIN == kSampleCi16) {
         const short2 s = static_cast<const short2 *>(g.x)[i];
-        v = make_float2((float)s.x, (float)s.y);
+        return make_float2((float)s.x, (float)s.y);
     } else
-        v = make_float2((float)static_cast<const short *>(g.x)[i], 0.f);
-    return from2<C>(v);
+        return make_float2((float)static_cast<const short *>(g.x)[i], 0.f);
+}
+template <uint32_t TIN, bool C> __device__ __forceinline__ Val<C> load_in(const IirLaunch &g, int32_t i)
+{
+    return from2<C>(chunk_sample<TIN>(g, i));
 }
 // ... or, below 0, a carried one
 template <uint32_t TIN, bool C> __device__ __forceinline__ Val<C> load_x(const IirLaunch &g, int32_t i)
 {
-    return i < 0 ? from2<C>(g.xh[(int32_t)g.nb - 1 + i]) : load_in<TIN, C>(g, i);
+    float2 v;
+    if (i < 0)
+        v = g.xh[(int32_t)g.nb - 1 + i];
+    else
+        v = chunk_sample<TIN>(g, i);
+    return from2<C>(v);
 }
 
 // acc + x b, the product as std::complex<float> rounds it. With a real
