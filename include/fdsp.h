@@ -287,7 +287,8 @@ int fdsp_iir_apply_device_noalloc(fdsp_iir_t h, const fdsp_cf32 *d_in, size_t n,
  * (reference src/transform/falcon_dsp_iir_filter.cc:104-396 per stream):
  * each stream's outputs equal the reference's sequential loop on that
  * stream, bit for bit up to the sign of zero, for every filter (the bank
- * runs one stream per GPU lane, so no filter needs the serial plan). Rows:
+ * runs the streams side by side on the GPU's lanes, so no filter needs the
+ * serial plan). Rows:
  * stream s's n samples at d_in + s * in_stride, its outputs at d_out + s *
  * out_stride (strides in samples, >= n); the host forms take n_streams
  * contiguous rows of n. Every stream advances by n samples per call; its
@@ -453,8 +454,9 @@ int fdsp_channelizer_get_tiling(fdsp_channelizer_t h, uint32_t *segment_len, uin
  *  - FDSP_KERNEL_SEGMENT_F32: the FDSP_CHAN_BATCHED default whenever every
  *    channel's window (taps per phase) is at most 64. One workgroup per input
  *    segment stages it once and computes every channel's outputs in it
- *    (groups of 2..8 channels with up 1, equal down and <= 32 taps on FP32
- *    matrix cores, the others on FP32 vector ALUs). Its tiling takes
+ *    (groups of 2..8 channels with up 1, equal down and <= 32 taps, and of 4..8
+ *    with 33..64 taps or discriminator tails, on FP32 matrix cores, the others
+ *    on FP32 vector ALUs). Its tiling takes
  *    segment_len a multiple of 256 from 1024 to 4096 (256 threads; default
  *    2560); the autotuner times 1024, 2048, 2560, 3072, 3584 and 4096.
  *  - FDSP_KERNEL_GROUPS_F32: the channel-group kernel in FP32 (windows

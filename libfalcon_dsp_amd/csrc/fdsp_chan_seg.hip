@@ -28,7 +28,8 @@
 //         real output in column 2c, its imaginary output in 2c+1. A sub-tile
 //         is 16 outputs of every channel of the group. Windows of 33 to 64
 //         taps take 32 K steps. Channels with a discriminator tail form groups
-//         of their own, whose sub-tiles overlap by one output.
+//         of their own, whose sub-tiles overlap by one output (both from four
+//         channels on).
 //   VALU  one channel (any up), window of at most 64 taps: one output per
 //         lane, taps zero-padded in front to kW = 32 or 64. With up 1 the taps
 //         are wavefront-uniform scalar loads; with up > 1 each lane reads the
